@@ -1481,29 +1481,30 @@ template <int HD>
 int attn_prefill_launch(const float* q, int ldq, const float* kc, const float* vc, int kv_dim,
                         int kv_mul, int heads, float* out, int ldo, int pos0, int n, hipStream_t st,
                         float* part = nullptr, char* planes = nullptr) {
-  // Head sizes 64 and 128 on the matrix cores (split products, fp16 or bf16;
-  // KL_PREFILL_ATTN=f32 keeps the fp32 products); 32 and 256 on the vector ALUs.
+  // Head sizes 64 and 128 on the matrix cores: split products for 128 and, over prepared planes,
+  // both (KL_PREFILL_ATTN=f32 keeps the fp32 products), fp32 products for 64; 32 and 256 on the
+  // vector ALUs.
   constexpr bool kMfma = HD == 64 || HD == 128;
   const char* env = kMfma ? std::getenv("KL_PREFILL_ATTN") : nullptr;  // read per launch (tests switch it)
-  const bool h2 = kMfma && !(env && std::strcmp(env, "f32") == 0);
-  const bool pre = h2 && planes;
-  const bool x6 = HD == 128 && h2 && !pre;
+  const bool split = kMfma && !(env && std::strcmp(env, "f32") == 0);
+  const bool pre = split && planes;
+  const bool x6 = HD == 128 && split && !pre;
   const int qh = pre && kv_mul % 2 == 0 ? 2 : 1;  // query heads per workgroup
-  const void* fn = qh == 2 ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, true, 2>)
-                   : pre ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, true, 1>)
+  const void* fn = qh == 2 ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, 2>)
+                   : pre ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, 1>)
                    : x6 ? reinterpret_cast<const void*>(&k_attn_prefill_x6)
-                   : h2 ? reinterpret_cast<const void*>(&k_attn_prefill_h2<64, false, 1>)
-                      : kMfma ? reinterpret_cast<const void*>(&k_attn_prefill_fa<kMfma ? HD : 64>)
-                              : reinterpret_cast<const void*>(&k_attn_prefill<HD>);
-  const size_t lds = x6 ? attn_prefill_x6_lds_bytes()
-                        : h2 ? attn_prefill_h2_lds_bytes(HD, pre)
-                        : kMfma ? attn_prefill_fa_lds_bytes(HD) : attn_prefill_lds_bytes(HD);
+                   : kMfma ? reinterpret_cast<const void*>(&k_attn_prefill_fa<kMfma ? HD : 64>)
+                           : reinterpret_cast<const void*>(&k_attn_prefill<HD>);
+  const size_t lds = pre ? attn_prefill_h2_lds_bytes(HD)
+                     : x6 ? attn_prefill_x6_lds_bytes()
+                     : kMfma ? attn_prefill_fa_lds_bytes(HD) : attn_prefill_lds_bytes(HD);
   static bool attr_set[4] = {false, false, false, false};  // per kernel of this head size
-  if (!attr_set[h2 + pre + qh - 1]) {
+  bool& attr = attr_set[qh == 2 ? 3 : pre ? 2 : x6 ? 1 : 0];
+  if (!attr) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                              static_cast<int>(lds));
     if (e != hipSuccess) return rc(e);
-    attr_set[h2 + pre + qh - 1] = true;
+    attr = true;
   }
   const float scale = 1.f / std::sqrt(static_cast<float>(HD));
   const dim3 grid((n + kPrefillQB - 1) / kPrefillQB, heads);
@@ -1525,17 +1526,12 @@ int attn_prefill_launch(const float* q, int ldq, const float* kc, const float* v
       const int r = launch_rc();
       if (r != KL_OK) return r;
       if (qh == 2)
-        hipLaunchKernelGGL((k_attn_prefill_h2<HD, true, 2>), dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc, kv_dim,
-                           kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
+        hipLaunchKernelGGL((k_attn_prefill_h2<HD, 2>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
       else
-        hipLaunchKernelGGL((k_attn_prefill_h2<HD, true, 1>), dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc, kv_dim,
-                           kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
+        hipLaunchKernelGGL((k_attn_prefill_h2<HD, 1>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
     } else if (x6)
       hipLaunchKernelGGL(k_attn_prefill_x6, dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc, kv_dim, kv_mul, out,
                          ldo, pos0, n, scale, heads, workers ? part : nullptr);
-    else if (h2)
-      hipLaunchKernelGGL((k_attn_prefill_h2<64, false, 1>), dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc, kv_dim,
-                         kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, nullptr, 0);
     else
       hipLaunchKernelGGL(k_attn_prefill_fa<HD>, dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc,
                          kv_dim, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr);
