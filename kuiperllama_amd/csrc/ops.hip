@@ -1490,12 +1490,12 @@ int attn_prefill_launch(const float* q, int ldq, const float* kc, const float* v
   const bool pre = split && planes;
   const bool x6 = HD == 128 && split && !pre;
   const int qh = pre && kv_mul % 2 == 0 ? 2 : 1;  // query heads per workgroup
-  const void* fn = qh == 2 ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, 2>)
-                   : pre ? reinterpret_cast<const void*>(&k_attn_prefill_h2<kMfma ? HD : 64, 1>)
+  const void* fn = qh == 2 ? reinterpret_cast<const void*>(&k_attn_prefill_planes<kMfma ? HD : 64, 2>)
+                   : pre ? reinterpret_cast<const void*>(&k_attn_prefill_planes<kMfma ? HD : 64, 1>)
                    : x6 ? reinterpret_cast<const void*>(&k_attn_prefill_x6)
                    : kMfma ? reinterpret_cast<const void*>(&k_attn_prefill_fa<kMfma ? HD : 64>)
                            : reinterpret_cast<const void*>(&k_attn_prefill<HD>);
-  const size_t lds = pre ? attn_prefill_h2_lds_bytes(HD)
+  const size_t lds = pre ? attn_prefill_planes_lds_bytes(HD)
                      : x6 ? attn_prefill_x6_lds_bytes()
                      : kMfma ? attn_prefill_fa_lds_bytes(HD) : attn_prefill_lds_bytes(HD);
   static bool attr_set[4] = {false, false, false, false};  // per kernel of this head size
@@ -1513,7 +1513,7 @@ int attn_prefill_launch(const float* q, int ldq, const float* kc, const float* v
     const unsigned blocks = workers ? workers : grid.x * grid.y / qh;
     if (pre) {
       const int nkb = (pos0 + n + kFaKB - 1) / kFaKB;
-      const size_t plds = attn_planes_block_bytes(HD) + 8 * sizeof(float);
+      const size_t plds = attn_planes_block_bytes(HD);
       static bool plds_set = false;
       if (!plds_set) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_planes<HD>),
@@ -1526,9 +1526,9 @@ int attn_prefill_launch(const float* q, int ldq, const float* kc, const float* v
       const int r = launch_rc();
       if (r != KL_OK) return r;
       if (qh == 2)
-        hipLaunchKernelGGL((k_attn_prefill_h2<HD, 2>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
+        hipLaunchKernelGGL((k_attn_prefill_planes<HD, 2>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
       else
-        hipLaunchKernelGGL((k_attn_prefill_h2<HD, 1>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
+        hipLaunchKernelGGL((k_attn_prefill_planes<HD, 1>), dim3(blocks), dim3(512), lds, st, q, ldq, kv_mul, out, ldo, pos0, n, scale, heads, workers ? part : nullptr, planes, nkb);
     } else if (x6)
       hipLaunchKernelGGL(k_attn_prefill_x6, dim3(blocks), dim3(512), lds, st, q, ldq, kc, vc, kv_dim, kv_mul, out,
                          ldo, pos0, n, scale, heads, workers ? part : nullptr);
@@ -1556,11 +1556,12 @@ size_t attn_planes_bytes(int keys, int kv_heads, int hd) {
              ? static_cast<size_t>(kv_heads) * ((keys + kFaKB - 1) / kFaKB) * attn_planes_block_bytes(hd) : 0;
 }
 
-// The pass over K and V costs a launch, 4 to 5 us, and 18 bytes per element of the cache;
-// it saves about 0.9 us of every key block that a workgroup walks.  Measured with 128-wide
-// heads: 95 key blocks per workgroup (12 heads, 4000 positions) 496 -> 411 + 8 us, 338 + 8 in pairs of heads, 4.5
-// (32 heads, 512 positions) 38.1 -> 33.0 + 5 us: taken from 8 on.  The bytes are
-// paid back where at least 16 row blocks of queries read a key block.
+// The pass over K and V costs a launch, 5 to 6 us, and 18 bytes per element of the cache; it saves
+// a part of every key block that a workgroup walks.  Measured per layer inside prompts without ->
+// with it, at 8 key blocks per workgroup: 12 heads of 64 (1152 positions) 42.9 -> 40.9 us, 32
+// of 64 (704) 49.8 -> 48.1, 12 of 128 (1152) 68.0 -> 66.2, 32 of 128 (1000, 16 blocks) 123 -> 122; at
+// 4.5 (32 heads of 128, 512 positions) the pass costs the 5 us that it saves: taken from 8 on.  The
+// bytes are paid back where at least 16 row blocks of queries read a key block.
 bool attn_planes_used(int pos0, int n, int heads, int kv_mul, int hd) {
   if (hd != 64 && hd != 128) return false;
   const FaGeom geo = fa_geom(pos0, n);
@@ -1570,8 +1571,8 @@ bool attn_planes_used(int pos0, int n, int heads, int kv_mul, int hd) {
 int attn_prefill_planes_run(int pos0, int n, int heads, int kv_mul, int hd, const float* q, int ldq,
                             const float* kc, const float* vc, int kv_dim, float* out, int ldo, void* ws,
                             size_t ws_bytes, char* planes, hipStream_t st) {
-  // From a position within a key block on, that block holds keys no row of the first row
-  // block attends; those stay out of its exponent only where the kernel itself splits.
+  // From a position within a key block on, a row block's last key block holds keys behind its last
+  // row: zeros times them are NaN where they are infinite, unless the kernel itself leaves them out.
   if (!planes || pos0 % kFaKB || !attn_planes_used(pos0, n, heads, kv_mul, hd))
     return kl_attn_prefill_ws(pos0, n, heads, kv_mul, hd, q, ldq, kc, vc, kv_dim, out, ldo, ws, ws_bytes, st);
   if (!ws || ws_bytes < (kv_mul % 2 == 0 ? 2 : 1) * attn_prefill_fa_ws_bytes(hd)) return KL_EWORKSPACE;
