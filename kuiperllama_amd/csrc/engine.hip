@@ -1198,13 +1198,13 @@ int kl_engine_create(const void* image, size_t bytes, int family, int quant, kl_
   }
   e->transform = family == KL_FAMILY_QWEN3 ? 2 : 1;
   {
-    // Split-product prefill GEMMs: every GEMM depth a multiple of 32, int8 in groups of
-    // 32 or more and rows that norm_h2_run takes (8192); KL_PREFILL_GEMM=f32 keeps the fp32
-    // matrix-core kernels, which any other int8 image runs.
+    // Split-product prefill GEMMs: every GEMM depth a multiple of 32, rows that norm_h2_run
+    // takes (8192), int8 in groups of 32 or more; KL_PREFILL_GEMM=f32 keeps the fp32
+    // matrix-core kernels, which any other image runs.
     const char* env = std::getenv("KL_PREFILL_GEMM");
-    e->pf_h2 = lay.D % 32 == 0 && lay.Dq % 32 == 0 && lay.F % 32 == 0 &&
+    e->pf_h2 = lay.D % 32 == 0 && lay.D <= 8192 && lay.Dq % 32 == 0 && lay.F % 32 == 0 &&
                !(env && std::strcmp(env, "f32") == 0) &&
-               (!quant || (lay.D <= 8192 && i8_packed_bytes(1, lay.D, lay.gs) && i8_packed_bytes(1, lay.Dq, lay.gs) &&
+               (!quant || (i8_packed_bytes(1, lay.D, lay.gs) && i8_packed_bytes(1, lay.Dq, lay.gs) &&
                            i8_packed_bytes(1, lay.F, lay.gs)));
   }
   int dev = 0;
