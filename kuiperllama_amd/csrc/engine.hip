@@ -1580,8 +1580,8 @@ int prefill_scratch(kl_engine* e, int rows) {
   r = kl_attn_prefill_workspace_size(rows, m.H, m.hd, &attn_ws);
   if (r != KL_OK) return r;
   if (m.H / m.KVH % 2 == 0) attn_ws *= 2;  // attn_prefill_planes_run takes heads in pairs
-  // Split-K partials: up to kPrefillMaxSplits x rows x D (the WO and W2
-  // outputs), and for int8 prompts of at most 32 rows also the grouped QKV
+  // Split-K partials of the fp32 matrix-core kernels (sized for in any case: prefill_planes may
+  // yet fall back on them): up to kPrefillMaxSplits x rows x D (the WO and W2 outputs), and for int8 prompts of at most 32 rows also the grouped QKV
   // and W1/W3 outputs at up to kPrefillMaxSplitsQ8 splits.
   size_t ws_floats = static_cast<size_t>(kPrefillMaxSplits) * R * m.D;
   // The split-product GEMMs choose up to 8 splits for WO and W2, 4 for the
@@ -1654,7 +1654,8 @@ void prefill_kv_planes(kl_engine* e, int keys, int rows) {
 }
 
 // Builds the GEMM operands of every layer's projections (once): fp32 as fp16 planes
-// with their row exponents, int8 packed.
+// with their row exponents, int8 packed.  Without memory for them this engine's prompts run
+// the fp32 matrix-core kernels from then on, which read the image's own weights.
 int prefill_planes(kl_engine* e) {
   if (e->xw_buf || !e->pf_h2) return KL_OK;
   const ImageLayout& m = e->lay;
@@ -1671,7 +1672,11 @@ int prefill_planes(kl_engine* e) {
   size_t per_layer = 0;
   for (int i = 0; i < 7; ++i) per_layer += bytes(i) + (q8 ? 0 : al(rows[i] * sizeof(int)));
   char* buf = nullptr;
-  if (hipMalloc(&buf, per_layer * m.L + al(nf * sizeof(unsigned))) != hipSuccess) return KL_ENOMEM;
+  if (hipMalloc(&buf, per_layer * m.L + al(nf * sizeof(unsigned))) != hipSuccess) {
+    (void)hipGetLastError();
+    e->pf_h2 = false;
+    return KL_OK;
+  }
   e->xw_buf = buf;
   hipStream_t hs = static_cast<hipStream_t>(e->stream);
   unsigned* flags = reinterpret_cast<unsigned*>(buf + per_layer * m.L);
