@@ -1817,7 +1817,7 @@ int prefill_chunk(kl_engine* e, int pos0, int n, int* pend_out) {
     }
     // attention_mha (llama3.cpp:651-669), then x += Wo . att
     PF(attn_prefill_planes_run(pos0, n, H, H / KVH, hd, e->pf_q, Dq, kc, vc, Dkv, e->pf_att, Dq, e->pf_aws,
-                               e->pf_aws_bytes, e->pf_kv, hs));
+                               e->pf_aws_bytes, e->pf_kv, e->pf_kv_keys, hs));
     // feed_forward (llama3.cpp:671-719)
     if (h2) {
       int dwo = 1, d13 = 1, d2 = 1;

@@ -127,15 +127,15 @@ int qkv_sum_rope_run(int style, int dim, int kv_dim, int hd, const float* ws, in
                      const float* bq, const float* bk, const float* bv, float* q, int ldq, float* k, int ldk,
                      float* v, int ldv, int pos0, int n, const float* sin_t, const float* cos_t,
                      hipStream_t st);
-// kl_attn_prefill_ws with K and V split into fp16 planes once, in front of the attention:
-// planes holds attn_planes_bytes of at least pos0 + n keys, ws twice
-// kl_attn_prefill_workspace_size's bytes where kv_mul is even.  Without planes, or for a call
-// that attn_planes_used turns away, kl_attn_prefill_ws itself.
+// kl_attn_prefill_ws with K and V split into planes once, in front of the attention:
+// planes holds attn_planes_bytes of planes_keys keys, ws twice
+// kl_attn_prefill_workspace_size's bytes where kv_mul is even.  Without planes for pos0 + n keys, or
+// for a call that attn_planes_used turns away, kl_attn_prefill_ws itself.
 size_t attn_planes_bytes(int keys, int kv_heads, int hd);
 bool attn_planes_used(int pos0, int n, int heads, int kv_mul, int hd);
 int attn_prefill_planes_run(int pos0, int n, int heads, int kv_mul, int hd, const float* q, int ldq,
                             const float* kc, const float* vc, int kv_dim, float* out, int ldo, void* ws,
-                            size_t ws_bytes, char* planes, hipStream_t st);
+                            size_t ws_bytes, char* planes, int planes_keys, hipStream_t st);
 // k_gemm_reduce over the outputs of g: C_s (+)= the sum of the split partials (+ bias).
 int gemm_reduce_run(const GemmArgs& g, hipStream_t st);
 

@@ -1570,10 +1570,10 @@ bool attn_planes_used(int pos0, int n, int heads, int kv_mul, int hd) {
 
 int attn_prefill_planes_run(int pos0, int n, int heads, int kv_mul, int hd, const float* q, int ldq,
                             const float* kc, const float* vc, int kv_dim, float* out, int ldo, void* ws,
-                            size_t ws_bytes, char* planes, hipStream_t st) {
+                            size_t ws_bytes, char* planes, int planes_keys, hipStream_t st) {
   // From a position within a key block on, a row block's last key block holds keys behind its last
   // row: zeros times them are NaN where they are infinite, unless the kernel itself leaves them out.
-  if (!planes || pos0 % kFaKB || !attn_planes_used(pos0, n, heads, kv_mul, hd))
+  if (!planes || pos0 + n > planes_keys || pos0 % kFaKB || !attn_planes_used(pos0, n, heads, kv_mul, hd))
     return kl_attn_prefill_ws(pos0, n, heads, kv_mul, hd, q, ldq, kc, vc, kv_dim, out, ldo, ws, ws_bytes, st);
   if (!ws || ws_bytes < (kv_mul % 2 == 0 ? 2 : 1) * attn_prefill_fa_ws_bytes(hd)) return KL_EWORKSPACE;
   float* part = static_cast<float*>(ws);
