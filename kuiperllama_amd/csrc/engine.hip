@@ -1885,6 +1885,12 @@ int kl_engine_prefill(kl_engine* e, const int32_t* prompt, int P, int32_t* next,
   if (r != KL_OK) return r;
   prefill_kv_planes(e, P, std::min(P, chunk));
   std::memcpy(e->xfer + kXferTok, prompt, sizeof(int32_t) * P);
+  // Launched kernels read the ids from e->xfer, which the next call writes: a call that fails
+  // waits for its own before it returns.
+  auto fail = [&](int code) {
+    (void)hipStreamSynchronize(e->stream);
+    return code;
+  };
   hipError_t err = prefill_ms ? hipEventRecord(e->ev0, e->stream) : hipSuccess;
   if (err != hipSuccess) return rc(err);
   int last_n = 0, pend = 0;
@@ -1904,11 +1910,11 @@ int kl_engine_prefill(kl_engine* e, const int32_t* prompt, int P, int32_t* next,
                  : kl_gemv_f32(e->pf_xlast, static_cast<const float*>(e->wcls.w), e->logits, m.V,
                                m.D, 1.f, e->stream);
   if (r == KL_OK) r = kl_argmax(e->logits, m.V, e->pf_next, e->pf_am, e->pf_am_bytes, e->stream);
-  if (r != KL_OK) return r;
+  if (r != KL_OK) return fail(r);
   if (prefill_ms) err = hipEventRecord(e->ev1, e->stream);
   if (err == hipSuccess) err = export_results(e, e->pf_next, logits);
   if (err == hipSuccess && prefill_ms) err = hipEventElapsedTime(prefill_ms, e->ev0, e->ev1);
-  if (err != hipSuccess) return rc(err);
+  if (err != hipSuccess) return fail(rc(err));
   if (next) *next = e->xfer[0];
   return KL_OK;
 }
