@@ -431,10 +431,17 @@ int kl_engine_bench(kl_engine* e, const int32_t* prompt, int P, int n_warmup, in
  * classifier and argmax of position P-1: *next (may be NULL) receives the
  * greedy token, logits (host, may be NULL) the vocab logits of position P-1.
  * Same result as P kl_engine_step calls up to float rounding; a following
- * kl_engine_step(e, *next, P, ...) continues the sequence.  Chunks of at most
- * 1024 positions.  KL_EUNSUPP for head sizes other than 32, 64, 128 (and for
- * int8 images whose dimensions are not whole 32-column blocks).  Blocks until
- * done; *prefill_ms (may be NULL) receives its device time. */
+ * kl_engine_step(e, *next, P, ...) continues the sequence.  Passes of at most
+ * 4096 positions (KL_PREFILL_CHUNK).  KL_EUNSUPP for head sizes other than 32, 64, 128
+ * and 256 (and for int8 images whose dimensions are not whole 32-column blocks).  Blocks until
+ * done; *prefill_ms (may be NULL) receives its device time.
+ * Operand range: the projections hold each activation row and each fp32 weight row (long
+ * prompts' attention each query and key row too) as two fp16 planes under the row's own power of two.
+ * Values down to 2^-16 of the row's largest keep 23 significand bits or more, smaller ones are held
+ * to 2^-39 of the row's largest: a product is as accurate as fp32 against the sizes of its two rows,
+ * not against its own terms where both rows spread over more than 2^16.  An infinity makes
+ * every product of its row NaN.  KL_PREFILL_GEMM=f32 and KL_PREFILL_ATTN=f32 in the environment
+ * keep fp32 products throughout. */
 int kl_engine_prefill(kl_engine* e, const int32_t* prompt, int P, int32_t* next, float* logits,
                       float* prefill_ms);
 /* When enabled (default off), kl_engine_generate runs prompts of 2 or more
