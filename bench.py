@@ -21,8 +21,8 @@ on both sides.  Prints one JSON line.
                  each of its launches in the profile steps
   prefill        the batched prompt prefill of cfg 5 (Qwen3-4B shape, 512
                  tokens) on the matrix cores: prompt tok/s, algorithmic
-                 TFLOP/s, the fraction of its matrix-core roofline (the
-                 split fp16 products at the fp16 peak), and the MFMA-busy fraction
+                 TFLOP/s, the fraction of its matrix-core roofline (the split
+                 products at the 16-bit peak), and the MFMA-busy fraction
                  rocprofv3 measured for the same command
                  (profiles/prefill_qwen3_4b_pmc.txt)
   configs        the other four BASELINE configs, each a short decode leg of
@@ -118,10 +118,12 @@ def measure_prefill(K, cfg, eng=None, reps: int = 3) -> dict:
     matrix cores would need at their peaks (bf16's is fp16's): fp32
     projections run as three fp16 products per multiply-add, int8 ones as two,
     or the weights' bytes (fp32: two fp16 planes) at 8 TB/s where that is
-    longer; the attention as three for the scores and four for the values
-    (head sizes 64 and 128); the classifier, and every product with
-    KL_PREFILL_GEMM=f32 or, for the attention, KL_PREFILL_ATTN=f32, at the
-    fp32 peak; `frac` = that time over the measured one."""
+    longer; the attention as six bf16 products (head size 128), or three fp16
+    ones for the scores and six bf16 ones for the values where K and V are split
+    once per layer (long prompts, head sizes 64 and 128); other attention, the
+    classifier, and every product with KL_PREFILL_GEMM=f32 or, for the
+    attention, KL_PREFILL_ATTN=f32, at the fp32 peak; `frac` = that time over
+    the measured one."""
     if eng is None:
         eng = K.Engine(K.synth_image(cfg), cfg)
     prompt = K.prompt_tokens(cfg)
@@ -143,8 +145,12 @@ def measure_prefill(K, cfg, eng=None, reps: int = 3) -> dict:
         proj_ms = max(products * proj / MFMA_BF16_PEAK_TFLOPS / 1e9, wbytes / HBM_PEAK_GBPS / 1e6)
     else:
         gemm, proj_ms = "fp32 MFMA" + (" (int8 dequantised)" if cfg.quant else ""), proj / MFMA_FP32_PEAK_TFLOPS / 1e9
-    attn_h2 = cfg.head_size in (64, 128) and os.environ.get("KL_PREFILL_ATTN") != "f32"
-    attn_ms = 3.5 * attn / MFMA_BF16_PEAK_TFLOPS / 1e9 if attn_h2 else attn / MFMA_FP32_PEAK_TFLOPS / 1e9
+    # K and V split once per layer: 8 key blocks of 64 per CU, 16 row blocks per key block.
+    nb = -(-P // 64)
+    planes = nb * (nb + 1) // 2 * cfg.heads >= 8 * 256 and nb * (cfg.heads // cfg.kv_heads) >= 16
+    split = cfg.head_size in (64, 128) and os.environ.get("KL_PREFILL_ATTN") != "f32"
+    products = 4.5 if split and planes else 6 if split and cfg.head_size == 128 else 0
+    attn_ms = products * attn / MFMA_BF16_PEAK_TFLOPS / 1e9 if products else attn / MFMA_FP32_PEAK_TFLOPS / 1e9
     roof_ms = proj_ms + attn_ms + cls / MFMA_FP32_PEAK_TFLOPS / 1e9
     return {"config": cfg.name, "tokens": P, "ms": round(ms, 3),
             "tok_s": round(P / (ms / 1e3), 1), "tflops": round(tf, 2), "flops": int(fl),
